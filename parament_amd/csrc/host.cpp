@@ -279,6 +279,7 @@ struct GradKey {
     double dt, hnorm;
     unsigned pts, amps, amps_set, dim, seg, chunk;
     int quad, ncoef, M, device, precision;
+    int manual;   // a manual order M and the table's same M take different polynomials (set_grad_scheme)
     GradKey() { memset(this, 0, sizeof(*this)); }
     bool operator==(const GradKey& o) const { return memcmp(this, &o, sizeof(*this)) == 0; }
 };
@@ -1879,7 +1880,7 @@ Parament_ErrorCode gradient(Context<R>* h, const cplx<R>* carr_dev, double dt, u
     key.E = E; key.V = V; key.W = W; key.dg = dg; key.aux = gsum;
     key.dt = dt; key.hnorm = h->hnorm; key.pts = pts; key.amps = amps; key.amps_set = h->amps; key.dim = h->dim;
     key.seg = h->ckpt_seg; key.chunk = h->ckpt_chunk; key.quad = h->quad; key.ncoef = h->ncoef; key.M = M;
-    key.device = h->device; key.precision = h->precision;
+    key.device = h->device; key.precision = h->precision; key.manual = h->manual ? 1 : 0;
     if (h->grad_exec && key == h->grad_key)
         return hipGraphLaunch(h->grad_exec, h->stream) == hipSuccess ? PARAMENT_STATUS_SUCCESS : PARAMENT_STATUS_CUBLAS_FAILED;
     if (!(key == h->grad_prev)) {   // first call with these arguments: launch directly
