@@ -19,6 +19,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../../include/parament.h"
+#include "buffer_set.hpp"
 #include "kernels.hpp"
 
 using pa::cplx;
@@ -330,7 +331,7 @@ template <class R> struct Context {
     C* d_c = nullptr; size_t cap_c = 0;
     void* d_leaves = nullptr; size_t cap_leaves = 0;
     void* d_nodes = nullptr; size_t cap_nodes = 0;
-    C* d_gen[5] = {}; size_t cap_gen = 0; int n_gen = 0;
+    pa::BufferSet gen;   // step-wise working arrays
     void* d_root = nullptr; size_t cap_root = 0;  // d x d result of the last equiprop
     char* pin = nullptr; bool pin_failed = false; // host-array calls: pinned controls, then the result (kPin*)
     void* d_c64 = nullptr; size_t cap_c64 = 0;    // complex64 contexts: controls widened to FP64
@@ -367,8 +368,7 @@ template <class R> void free_working(Context<R>* h) {
     hipFree(h->d_c); h->d_c = nullptr; h->cap_c = 0;
     hipFree(h->d_leaves); h->d_leaves = nullptr; h->cap_leaves = 0;
     hipFree(h->d_nodes); h->d_nodes = nullptr; h->cap_nodes = 0;
-    for (auto& p : h->d_gen) { hipFree(p); p = nullptr; }
-    h->cap_gen = 0; h->n_gen = 0;
+    h->gen.clear([](void* p) { hipFree(p); });
     hipFree(h->d_root); h->d_root = nullptr; h->cap_root = 0;
     if (h->pin) { hipHostFree(h->pin); h->pin = nullptr; }
     hipFree(h->d_c64); h->d_c64 = nullptr; h->cap_c64 = 0;
@@ -821,28 +821,28 @@ int gemm_mode_of(int precision) {
 
 constexpr int kLowTreeLevels = 3;   // tree levels run in the low-precision products
 
-// n (3 .. 5) step-wise working arrays of `bytes` each: the context's, grown together, or pieces of a
-// fixed workspace (which is left as it was when they do not fit).
-template <class R> bool gen_buffers(Context<R>* h, Workspace& ws, size_t bytes, void* out[], int n = 3) {
+// Step-wise working arrays of `bytes` each, the context's or pieces of a fixed workspace: want of them, or need
+// where memory does not hold want.  The number taken, 0 when need do not fit either.
+template <class R> int gen_buffers(Context<R>* h, Workspace& ws, size_t bytes, int need, int want, void* out[]) {
     if (ws.fixed) {
         const size_t used = ws.used;
-        for (int i = 0; i < n; ++i)
-            if (!(out[i] = ws.get(nullptr, nullptr, bytes))) { ws.used = used; return false; }
-        return true;
+        for (int n = want;; n = need) {
+            int i = 0;
+            ws.used = used;
+            while (i < n && (out[i] = ws.get(nullptr, nullptr, bytes))) ++i;
+            if (i == n || n == need) return i == n ? n : 0;
+        }
     }
-    if (h->cap_gen < bytes || h->n_gen < n) {
-        for (auto& p : h->d_gen) { hipFree(p); p = nullptr; }
-        h->cap_gen = 0; h->n_gen = 0;
-        for (int i = 0; i < n; ++i)
-            if (hipMalloc(&h->d_gen[i], bytes) != hipSuccess) {
-                hipGetLastError();
-                for (auto& q : h->d_gen) { hipFree(q); q = nullptr; }
-                return false;
-            }
-        h->cap_gen = bytes; h->n_gen = n;
-    }
-    for (int i = 0; i < n; ++i) out[i] = h->d_gen[i];
-    return true;
+    const int n = h->gen.get(
+        bytes, need, want,
+        [](size_t b) {
+            void* p = nullptr;
+            if (hipMalloc(&p, b) != hipSuccess) { hipGetLastError(); p = nullptr; }
+            return p;
+        },
+        [](void* p) { hipFree(p); });
+    for (int i = 0; i < n; ++i) out[i] = h->gen.p[i];
+    return n;
 }
 
 // Step-wise form (any dim): the Clenshaw GEMMs (or the power form's) batched over all slices on
@@ -859,7 +859,8 @@ Parament_ErrorCode run_mixed_stepwise(Context<R>* h, const MixedSrc& m, double2*
     const int mode = f16 ? pa::GEMM_F16X2 : gemm_mode_of(h->precision);
     hipStream_t st = h->stream;
     void* gen[4] = {nullptr, nullptr, nullptr, nullptr};
-    if (!gen_buffers(h, ws, (size_t)N * dd * sizeof(float2), gen, power && M >= 7 ? 4 : 3)) return ws.failure();
+    const int need = power && M >= 7 ? 4 : 3;
+    if (!gen_buffers(h, ws, (size_t)N * dd * sizeof(float2), need, need, gen)) return ws.failure();
     double are[pa::kMaxCheb], aim[pa::kMaxCheb];
     bessel(M, m.tau * h->hnorm, are, aim);
     pa::ChebArgs<double> ca;
@@ -1174,8 +1175,10 @@ Parament_ErrorCode run(Context<R>* h, const cplx<R>* carr_dev, double dt, unsign
     const bool power = sizeof(R) == 4 && stepwise_power(M, tau * h->hnorm);
     void* gen[5] = {};
     PolyScheme ps = stepwise_scheme<R>(M, tau * h->hnorm, h->manual);
-    if (ps.deg && !gen_buffers(h, ws, (size_t)N * dd * sizeof(C), gen, poly_buffers(ps))) ps = PolyScheme();
-    if (!ps.deg && !gen_buffers(h, ws, (size_t)N * dd * sizeof(C), gen, power && M >= 7 ? 4 : 3)) return ws.failure();
+    const int need = power && M >= 7 ? 4 : 3, want = ps.deg ? poly_buffers(ps) : need;
+    const int got = gen_buffers(h, ws, (size_t)N * dd * sizeof(C), need, want, gen);
+    if (!got) return ws.failure();
+    if (got < want) ps = PolyScheme();
     C* X = reinterpret_cast<C*>(gen[0]);
     C* w1 = reinterpret_cast<C*>(gen[1]);
     C* w2 = reinterpret_cast<C*>(gen[2]);
@@ -1246,7 +1249,7 @@ Parament_ErrorCode run_replayable(Context<R>* h, const cplx<R>* carr_dev, double
     PropKey key;
     key.carr = carr_dev; key.out = out_dev; key.ops = h->d_ops; key.ops64 = h->d_ops64; key.opsP = h->d_opsP;
     key.leaves = h->d_leaves; key.nodes = h->d_nodes; key.c64 = h->d_c64;
-    for (int i = 0; i < 5; ++i) key.gen[i] = h->d_gen[i];
+    for (int i = 0; i < 5; ++i) key.gen[i] = h->gen.p[i];
     key.out64 = h->d_out64; key.stream = h->stream;
     key.dt = dt; key.hnorm = h->hnorm; key.pts = pts; key.amps = amps; key.amps_set = h->amps; key.dim = h->dim;
     key.quad = h->quad; key.magnus = h->magnus ? 1 : 0; key.ncoef = h->ncoef; key.precision = h->precision;
