@@ -27,6 +27,8 @@
 // to 335 us.
 #include "kernels.hpp"
 
+#include <type_traits>
+
 namespace pa {
 
 namespace {
@@ -200,8 +202,14 @@ __device__ __forceinline__ double2 coef_finish_h(const Controls<double>& q, cons
 // combine returns unchanged bit for bit (the reference's odd carry).
 // Node w of the problem a: its 2^F slices and their product.  cur: first plane set of the pair the next product's operands go to
 // (kept by the caller from one problem to the next: waves may still read the other pair).
-template <int D, int F, int FULL, int SCHEME>
-__device__ __forceinline__ void h2_node(const MixedArgs& a, _Float16* planes, double2* coef, int& cur, int w) {
+//
+// CHECK: values beyond fp16's range are met (controls of any modulus, slices far from unitary).  They become
+// infinities in their product and reach the node as these or as NaNs, so a node that is not finite is not stored and
+// the result is false.  F32: the node with FP32 products instead (S = 1, two plane pairs of FP32, a barrier on
+// either side of a product), for such nodes.
+template <int D, int F, int FULL, int SCHEME, bool CHECK = false, bool F32 = false>
+__device__ __forceinline__ bool h2_node(const MixedArgs& a, _Float16* planes, double2* coef, int& cur, int w) {
+    constexpr float S = F32 ? 1.0f : kScale, inv = 1.0f / S;
     constexpr int G = HShape<D>::G, PL = HShape<D>::PL, WC = HShape<D>::WC;
     constexpr int TN = HShape<D>::TN;
     constexpr int NB = 1 << F;
@@ -222,9 +230,43 @@ __device__ __forceinline__ void h2_node(const MixedArgs& a, _Float16* planes, do
     float one = 1.0f;   // opaque to the compiler (split2s)
     asm volatile("" : "+v"(one));
     auto set = [&](int k) { return planes + cur + 4 * PL * k; };
-    auto flip = [&]() { cur = 8 * PL - cur; };
+    constexpr int SF = D + 2, PF = D * SF;
+    static_assert(4 * PF * sizeof(float) <= 16 * PL * sizeof(_Float16), "the FP32 planes fit in the others' place");
+    float* fp = reinterpret_cast<float*>(planes);
+    // operand k = 0, 1 of the next product; lead: its leading part is enough
+    auto put = [&](const Tile& t, int k, auto lead) {
+        if constexpr (F32) {
+#pragma unroll
+            for (int n = 0; n < TN; ++n)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int at = 2 * k * PF + hrow(row0, v) * SF + hcol(col0, n);
+                    fp[at] = t.re[n][v]; fp[PF + at] = t.im[n][v];
+                }
+        } else {
+            write_h2<D, decltype(lead)::value ? 1 : 2>(t, set(k), row0, col0, one);
+        }
+    };
+    // the product of operands k1 and k2, after a barrier; the next one's may be put at once
+    auto product = [&](int k1, int k2, Tile& c, auto lead) {
+        if constexpr (F32) {
+            CTile<float, 1, TN> t;
+            wave_cgemm<float, 1, TN, D, SF, SF>(fp + 2 * k1 * PF, fp + (2 * k1 + 1) * PF, fp + 2 * k2 * PF,
+                                                fp + (2 * k2 + 1) * PF, row0, col0, t);
+#pragma unroll
+            for (int n = 0; n < TN; ++n)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) { c.re[n][v] = t.re[0][n][v]; c.im[n][v] = t.im[0][n][v]; }
+            __syncthreads();
+        } else {
+            wave_cgemm_h2<D, decltype(lead)::value ? 1 : FULL>(set(k1), set(k2), row0, col0, c);
+            cur = 8 * PL - cur;
+        }
+    };
+    constexpr std::false_type full{};
+    constexpr std::true_type lead{};
     // the assembly forms S Z = -i tau S H0 + sum_t (-i tau S c'_t) O_t: coef[] holds -i tau S c'_t
-    const double ts = a.ctl.tau * (double)kScale;
+    const double ts = a.ctl.tau * (double)S;
     auto scaled = [&](double2 c) { return mk<double>(c.y * ts, -c.x * ts); };
     auto slice = [&](int j, int jn, Tile& e) __attribute__((always_inline)) {
         if (!coef_ready) {
@@ -287,19 +329,18 @@ __device__ __forceinline__ void h2_node(const MixedArgs& a, _Float16* planes, do
                 zl.re[n][v] = (float)(x[v].x - (double)yr); zl.im[n][v] = (float)(x[v].y - (double)yi);
             }
         }
-        write_h2<D>(z, set(0), row0, col0, one);
+        put(z, 0, full);
         __syncthreads();
         const bool pre = prefetch && jn >= 0 && jn < a.N;
         RawCoefH raw;
         if (pre && tid < a.ncoef) raw = coef_load_h(a.ctl, tid, jn);
         Tile z2, p, acc;
-        wave_cgemm_h2<D, FULL>(set(0), set(0), row0, col0, acc);   // Z Z
-        flip();
+        product(0, 0, acc, full);   // Z Z
         auto unscale = [&](Tile& t) {
 #pragma unroll
             for (int n = 0; n < TN; ++n)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) { t.re[n][v] = acc.re[n][v] * kInvScale; t.im[n][v] = acc.im[n][v] * kInvScale; }
+                for (int v = 0; v < 4; ++v) { t.re[n][v] = acc.re[n][v] * inv; t.im[n][v] = acc.im[n][v] * inv; }
         };
         unscale(z2);
         auto publish = [&]() {   // the operands stored above become readable
@@ -317,11 +358,10 @@ __device__ __forceinline__ void h2_node(const MixedArgs& a, _Float16* planes, do
                     t.re[n][v] = __builtin_fmaf(q3, z2.re[n][v], z.re[n][v]);
                     t.im[n][v] = __builtin_fmaf(q3, z2.im[n][v], z.im[n][v]);
                 }
-            write_h2<D>(z2, set(0), row0, col0, one);
-            write_h2<D>(t, set(1), row0, col0, one);
+            put(z2, 0, full);
+            put(t, 1, full);
             publish();
-            wave_cgemm_h2<D, FULL>(set(0), set(1), row0, col0, acc);   // P = Z2 (Z + q3 Z2)
-            flip();
+            product(0, 1, acc, full);   // P = Z2 (Z + q3 Z2)
             unscale(p);
             Tile u;
 #pragma unroll
@@ -335,61 +375,60 @@ __device__ __forceinline__ void h2_node(const MixedArgs& a, _Float16* planes, do
                     rest.re[n][v] = __builtin_fmaf(q8, p.re[n][v], __builtin_fmaf(q7, p.re[n][v], __builtin_fmaf(q2, z2.re[n][v], 0.5f * z2.re[n][v])));
                     rest.im[n][v] = __builtin_fmaf(q8, p.im[n][v], __builtin_fmaf(q7, p.im[n][v], __builtin_fmaf(q2, z2.im[n][v], 0.5f * z2.im[n][v])));
                 }
-            write_h2<D>(u, set(0), row0, col0, one);
-            write_h2<D>(t, set(1), row0, col0, one);
+            put(u, 0, full);
+            put(t, 1, full);
             __syncthreads();
-            wave_cgemm_h2<D, FULL>(set(0), set(1), row0, col0, acc);
-            flip();
+            product(0, 1, acc, full);
+            const float zw = F32 ? a.zw * kScale : a.zw;
 #pragma unroll
             for (int n = 0; n < TN; ++n)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    rest.re[n][v] = __builtin_fmaf(a.zw, acc.re[n][v], rest.re[n][v]);
-                    rest.im[n][v] = __builtin_fmaf(a.zw, acc.im[n][v], rest.im[n][v]);
+                    rest.re[n][v] = __builtin_fmaf(zw, acc.re[n][v], rest.re[n][v]);
+                    rest.im[n][v] = __builtin_fmaf(zw, acc.im[n][v], rest.im[n][v]);
                 }
         } else {
             // Q_j = c_2j I + c_2j+1 Z + Z2 Q_j+1 for j = J .. 1, without c_2 I in Q_1; each Q_j's planes go
             // beside a copy of Z2's, so that both operands of a product lie in its pair
             const int J = (M - 1) / 2;
-            auto lead_only = [&](int jj) { return jj >= 1 && ((a.ps_levels >> (2 * jj)) & 3) == 0; };
+            auto lead_only = [&](int jj) { return !CHECK && !F32 && jj >= 1 && ((a.ps_levels >> (2 * jj)) & 3) == 0; };
             Tile q;
             for (int jj = J; jj >= 1; --jj) {
-                const float cd = jj > 1 ? a.zc[2 * jj] * kScale : 0.f, cz = a.zc[2 * jj + 1], cl = jj == 1 ? a.zw : 0.f;
+                const float cd = jj > 1 ? a.zc[2 * jj] * S : 0.f, cz = a.zc[2 * jj + 1], cl = jj == 1 ? a.zw : 0.f;
 #pragma unroll
                 for (int n = 0; n < TN; ++n)
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
-                        const float br = jj < J ? acc.re[n][v] * kInvScale : 0.f;
-                        const float bi = jj < J ? acc.im[n][v] * kInvScale : 0.f;
+                        const float br = jj < J ? acc.re[n][v] * inv : 0.f;
+                        const float bi = jj < J ? acc.im[n][v] * inv : 0.f;
                         q.re[n][v] = __builtin_fmaf(cl, z.re[n][v], __builtin_fmaf(cz, z.re[n][v], br + (dg[n][v] ? cd : 0.f)));
                         q.im[n][v] = __builtin_fmaf(cl, z.im[n][v], __builtin_fmaf(cz, z.im[n][v], bi));
                     }
                 if (lead_only(jj - 1)) {
-                    write_h2<D, 1>(z2, set(0), row0, col0, one);
-                    write_h2<D, 1>(q, set(1), row0, col0, one);
+                    put(z2, 0, lead);
+                    put(q, 1, lead);
                 } else {
-                    write_h2<D>(z2, set(0), row0, col0, one);
-                    write_h2<D>(q, set(1), row0, col0, one);
+                    put(z2, 0, full);
+                    put(q, 1, full);
                 }
                 if (jj == J) publish();
                 else __syncthreads();
-                if (lead_only(jj - 1)) wave_cgemm_h2<D, 1>(set(0), set(1), row0, col0, acc);
-                else wave_cgemm_h2<D, FULL>(set(0), set(1), row0, col0, acc);
-                flip();
+                if (lead_only(jj - 1)) product(0, 1, acc, lead);
+                else product(0, 1, acc, full);
             }
             const float q2 = a.zc[2];
 #pragma unroll
             for (int n = 0; n < TN; ++n)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    rest.re[n][v] = __builtin_fmaf(q2, z2.re[n][v], __builtin_fmaf(0.5f, z2.re[n][v], acc.re[n][v] * kInvScale));
-                    rest.im[n][v] = __builtin_fmaf(q2, z2.im[n][v], __builtin_fmaf(0.5f, z2.im[n][v], acc.im[n][v] * kInvScale));
+                    rest.re[n][v] = __builtin_fmaf(q2, z2.re[n][v], __builtin_fmaf(0.5f, z2.re[n][v], acc.re[n][v] * inv));
+                    rest.im[n][v] = __builtin_fmaf(q2, z2.im[n][v], __builtin_fmaf(0.5f, z2.im[n][v], acc.im[n][v] * inv));
                 }
         }
         coef_ready = pre;
         // E = c_0' I + Z + (c_1 - 1) Z + rest, Z = z + zl: what is added to z is below z in size, and the
         // sum is rounded once
-        const float e0 = a.zc[0] * kScale, e1 = a.zc[1];
+        const float e0 = a.zc[0] * S, e1 = a.zc[1];
 #pragma unroll
         for (int n = 0; n < TN; ++n)
 #pragma unroll
@@ -402,18 +441,17 @@ __device__ __forceinline__ void h2_node(const MixedArgs& a, _Float16* planes, do
 
     // A := A + B + A B for the later node A and the earlier node B (in place; both held scaled by S)
     auto combine = [&](Tile& A, const Tile& B) __attribute__((always_inline)) {
-        write_h2<D>(A, set(0), row0, col0, one);
-        write_h2<D>(B, set(1), row0, col0, one);
+        put(A, 0, full);
+        put(B, 1, full);
         __syncthreads();
         Tile acc;
-        wave_cgemm_h2<D, FULL>(set(0), set(1), row0, col0, acc);
-        flip();
+        product(0, 1, acc, full);
 #pragma unroll
         for (int n = 0; n < TN; ++n)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                A.re[n][v] = __builtin_fmaf(acc.re[n][v], kInvScale, A.re[n][v] + B.re[n][v]);
-                A.im[n][v] = __builtin_fmaf(acc.im[n][v], kInvScale, A.im[n][v] + B.im[n][v]);
+                A.re[n][v] = __builtin_fmaf(acc.re[n][v], inv, A.re[n][v] + B.re[n][v]);
+                A.im[n][v] = __builtin_fmaf(acc.im[n][v], inv, A.im[n][v] + B.im[n][v]);
             }
     };
 
@@ -443,6 +481,14 @@ __device__ __forceinline__ void h2_node(const MixedArgs& a, _Float16* planes, do
             }
         }
         if (carry) {   // p = 2^F - 1: e is the block's node
+            if constexpr (CHECK) {
+                bool lost = false;
+#pragma unroll
+                for (int n = 0; n < TN; ++n)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) lost |= !(fabsf(e.re[n][v]) + fabsf(e.im[n][v]) < INFINITY);
+                if (__syncthreads_or(lost)) return false;
+            }
             float2* out = a.out + (size_t)w * dd;
 #pragma unroll
             for (int n = 0; n < TN; ++n) {
@@ -450,10 +496,11 @@ __device__ __forceinline__ void h2_node(const MixedArgs& a, _Float16* planes, do
 #pragma unroll
                 for (int v = 0; v < 4; ++v)
                     if (i + v < d && k < d)
-                        out[(i + v) * d + k] = make_float2(e.re[n][v] * kInvScale, e.im[n][v] * kInvScale);
+                        out[(i + v) * d + k] = make_float2(e.re[n][v] * inv, e.im[n][v] * inv);
             }
         }
     }
+    return true;
 }
 
 template <int D, int F, int FULL, int SCHEME>
@@ -466,7 +513,8 @@ __global__ __launch_bounds__(64 * HShape<D>::G, 2) void cheb_h2_kernel(MixedArgs
 }
 
 // Nodes of many problems (an ensemble's dim class): task (i, w) is node w of inst[i], whose arguments stay
-// in memory and are read as scalars.  16 systems of dims 33-64 with 1,000-4,000 slices take 1.38 ms with it
+// in memory and are read as scalars.  A node whose values leave fp16's range is formed again in FP32 products; those on
+// leading parts only, which rest on controls of modulus 1, are not used.  16 systems of dims 33-64 with 1,000-4,000 slices take 1.38 ms with it
 // against 2.42 ms on the FP32 slice kernel and its two lowest tree levels.
 template <int D, int F, int FULL, int SCHEME>
 __global__ __launch_bounds__(64 * HShape<D>::G, 2) void ens_h2_kernel(const MixedArgs* __restrict__ inst,
@@ -476,7 +524,8 @@ __global__ __launch_bounds__(64 * HShape<D>::G, 2) void ens_h2_kernel(const Mixe
     int cur = 0;
     for (int t = blockIdx.x; t < ntasks; t += gridDim.x) {
         const int2 tk = tasks[t];
-        h2_node<D, F, FULL, SCHEME>(inst[tk.x], planes, coef, cur, tk.y);
+        if (!h2_node<D, F, FULL, SCHEME, true>(inst[tk.x], planes, coef, cur, tk.y))
+            h2_node<D, F, FULL, SCHEME, false, true>(inst[tk.x], planes, coef, cur, tk.y);
     }
 }
 

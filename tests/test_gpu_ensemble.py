@@ -284,3 +284,39 @@ def test_ensemble_split_slices(xs, pts):
         ref = eo.equiprop(h0, hk, c32, dt[i])
         assert rel_err(first[i], ref) < 1e-5 + 2.0 ** -23 * pts[i] * (x[i] + 0.05), (dims[i], pts[i], x[i])
         assert np.array_equal(first[i], again[i])
+
+
+@pytest.mark.parametrize("others", [12, 4100])   # no folded tree levels; three
+@pytest.mark.parametrize("kind", ["strong", "far", "gain"])
+@pytest.mark.parametrize("x, m", [(0.2, 5), (0.4, 7), (0.9, 9)])
+def test_ensemble_values_beyond_fp16(x, m, kind, others):
+    """Slices of norm 2.2 and 6 (controls far above modulus 1) and non-unitary ones (imaginary controls of
+    modulus 1), whose products leave fp16's range at the split kernel's usual scale: as far from the
+    exponentials as the degree-M polynomial is.  Per slice up to six products of relative error 2^-22, terms up to 20
+    times their sum (e^6 against the polynomial's value), twelve slices: 20 * 72 * 2^-22 = 3.4e-4, below 1e-3."""
+    from oracle.expm_stepwise import expm_stepwise
+    from parament_amd.ensemble import Ensemble
+    rng = np.random.default_rng(17)
+    dims, hs, cs, dt, pts = [17, 32, 33, 48, 49, 64], [], [], [], []
+    for i, d in enumerate(dims):
+        h = [0.1 * gue(rng, d), np.diag(rng.choice([-1.0, 1.0], d)) + 0j]
+        n = 12 if i % 2 == 0 else others
+        r = {"strong": 2.2, "far": 6.0, "gain": x}[kind] if i % 2 == 0 else x
+        hn = eo.hamiltonian_norm(h[0], h[1:])
+        a = (r * hn / x if kind != "gain" else 1j if i % 2 == 0 else 1.0) * rng.uniform(0.9, 1.0, (1, n))
+        hs.append(h); cs.append(a); dt.append(x / hn); pts.append(n)
+    with Ensemble(dims, [1] * 6, pts, dt, "none") as e:
+        e.set_hamiltonians(hs)
+        us = e.equiprop(cs)
+    for i, (h, c, u) in enumerate(zip(hs, cs, us)):
+        h0, hk, c32 = as_c64_inputs(h[0], h[1:], c)
+        ref = eo.equiprop(h0, hk, c32, dt[i], cycles=m)
+        assert np.all(np.isfinite(u)), dims[i]
+        if i % 2 == 0:
+            exact = expm_stepwise(h0, hk, c32, dt[i])
+            scale = np.linalg.norm(ref)
+            assert np.linalg.norm(u - exact) < 1.1 * np.linalg.norm(ref - exact) + 1e-3 * scale, dims[i]
+            if m != 7:   # exactly the degree-M polynomial
+                assert rel_err(u, ref) < 1e-3, dims[i]
+        else:
+            assert rel_err(u, ref) < 2e-5 + 2.0 ** -23 * pts[i] * x, dims[i]
