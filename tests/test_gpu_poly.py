@@ -200,3 +200,23 @@ def test_complex128_tiles(d, n):
         p.set_gradient_checkpointing(0, 8)
         f8, g8 = p.gate_fidelity_gradient(dt, *c, target=target)
     assert abs(f - f8) < 1e-12 and rel_err(g, g8) < 1e-12
+
+
+@pytest.mark.parametrize("x, m", [(0.4, 7), (0.9, 9)])
+@pytest.mark.parametrize("d, n", [(2, 300), (40, 33), (65, 2), (100, 33)])
+def test_complex64_stepwise_is_the_power_form(x, m, d, n):
+    """The FP32 step-wise path evaluates the degree-M polynomial in powers of tau X whether M is the table's
+    choice or set by hand, bit for bit (the product-saving schemes are less accurate in FP32)."""
+    import parament_amd as parament
+    h0, hks, c, dt = problem(d, 2, n, x, False)
+    us = []
+    for manual in (False, True):
+        with parament.Parament("fp32") as p:
+            p.set_kernel_path("stepwise")
+            p.set_precision_mode("native")
+            if manual:
+                p.set_iteration_cycles(m)
+            p.set_hamiltonian(h0, *hks)
+            us.append(p.equiprop(dt, *c))
+            assert p.iteration_cycles == m
+    assert np.array_equal(*us)
