@@ -540,13 +540,15 @@ inline PolyScheme auto_scheme(int M, double x, bool manual, bool exact = false) 
     return poly_scheme(M <= 7 ? 8 : 12, x, false, exact);
 }
 
-// The gradient's slices and derivative take it from M = 7 on (at M = 5 the power form takes as many passes),
-// with exact Bessel values: its power form, too, rounds c_0 to 1 (at dim 32, 4,096 slices the reference's
+// The gradient's slices and derivative take it from M = 7 on (at M = 5 the power form takes as many passes), in
+// complex64 at M = 7 only (at M = 9 the degree-12 scheme in FP32 gave dF/dc at dims 16-32 1.09 times the power form's
+// error), with exact Bessel values: its power form, too, rounds c_0 to 1 (at dim 32, 4,096 slices the reference's
 // values' c_0 - 1 = 5e-17 would take the error of F and dF from 2e-15 to 4e-13).
 template <class R> void set_grad_scheme(pa::ChebArgs<R>& ca, double x, bool manual) {
     if (ca.M < 7) return;
-    const PolyScheme ps =
-        sizeof(R) == 4 && ca.M == 7 && !manual && power_form_ok(12, x) ? poly_scheme(8, x, true, true) : auto_scheme(ca.M, x, manual, true);
+    PolyScheme ps;
+    if (sizeof(R) == 8) ps = auto_scheme(ca.M, x, manual, true);
+    else if (ca.M == 7 && !manual && power_form_ok(12, x)) ps = poly_scheme(8, x, true, true);
     ca.pdeg = ps.deg;
     for (int k = 0; k < pa::kPolyCoeffs; ++k) ca.pc[k] = (R)ps.q[k];
 }

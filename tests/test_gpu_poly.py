@@ -220,3 +220,22 @@ def test_complex64_stepwise_is_the_power_form(x, m, d, n):
             us.append(p.equiprop(dt, *c))
             assert p.iteration_cycles == m
     assert np.array_equal(*us)
+
+
+@pytest.mark.parametrize("d, n", [(5, 40), (16, 1), (32, 9)])
+def test_complex64_gradient_keeps_the_power_form(d, n):
+    """At M = 9 the complex64 gradient evaluates the degree-9 polynomial in powers of tau X whether M is the
+    table's choice or set by hand, bit for bit."""
+    import parament_amd as parament
+    from parament_amd.workloads import haar_unitary
+    h0, hks, c, dt = problem(d, 2, n, 0.9, False)
+    t = haar_unitary(np.random.default_rng(d), d)
+    res = []
+    for manual in (False, True):
+        with parament.Parament("fp32") as p:
+            if manual:
+                p.set_iteration_cycles(9)
+            p.set_hamiltonian(h0, *hks)
+            res.append(p.gate_fidelity_gradient(dt, *c, target=t))
+            assert p.iteration_cycles == 9
+    assert res[0][0] == res[1][0] and np.array_equal(res[0][1], res[1][1])
