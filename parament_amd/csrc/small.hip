@@ -114,7 +114,9 @@ __device__ __forceinline__ void wave_order() {
 
 constexpr int kTinyFold = 5;   // most tree levels a wave folds one slice after another
 
-// NC: operators after H0 held in registers for the launch (0: any number, from LDS).  SCHEME 0: the
+// NC: operators after H0 held in registers for the launch (0: any number, from LDS, with each coefficient
+// evaluated by one lane and handed to its slice's lanes through LDS; evaluated by every lane, 64 of them took 87 us at
+// 4,096 slices of dim 5, complex128, and 47 so).  SCHEME 0: the
 // recurrence; 8, 12: poly_slice_tile's schemes (complex128).
 template <class R, int BD, int NC, int SCHEME>
 __global__ __launch_bounds__(1024) void tiny_kernel(ChebArgs<R> a, int F, int final_level) {
@@ -126,7 +128,8 @@ __global__ __launch_bounds__(1024) void tiny_kernel(ChebArgs<R> a, int F, int fi
     C* lds = reinterpret_cast<C*>(tiny_lds);
     const T L;
     const int W = blockDim.x >> 6, wave = threadIdx.x >> 6, d = a.d, dd = d * d;
-    // per wave: NS matrices as first operands, NS as second ones; then (NC = 0) the operators
+    // per wave: NS matrices as first operands, NS as second ones; then (NC = 0) the operators and, per wave, 64
+    // coefficients
     C* const s0 = lds + (size_t)wave * 2 * NS * SL + L.q * SL;
     C* const s1 = s0 + NS * SL;
     C* const ops = lds + (size_t)W * 2 * NS * SL;
@@ -169,6 +172,17 @@ __global__ __launch_bounds__(1024) void tiny_kernel(ChebArgs<R> a, int F, int fi
             next[t] = j < a.N ? slice_coefficient(a.ctl, t, a.j0 + (int)j) : mk<R>(0, 0);
     };
     prefetch(j0);
+    // NC = 0: lane l evaluates coefficients PER r + l % PER, r = 0, 1, .., of the wave's node l / PER
+    constexpr int PER = 64 / NS;
+    const int lane = threadIdx.x & 63, mine = lane % PER;
+    const long jm = (long)((blockIdx.x * W + wave) * NS + lane / PER) << F;
+    const int live = (int)min(max(a.N - jm, 0l), 1l << F);   // slices of that node
+    C* const cf = ops + a.ncoef * dd + wave * 64;
+    auto evaluate = [&](int t, int p) {
+        return t < a.ncoef && p < live ? slice_coefficient(a.ctl, t, a.j0 + (int)jm + p) : mk<R>(0, 0);
+    };
+    C ahead = mk<R>(0, 0);
+    if constexpr (NC == 0) ahead = evaluate(mine, 0);
     Tile pend[kTinyFold], e;
 #pragma unroll 1
     for (int p = 0; p < (1 << F); ++p) {
@@ -183,11 +197,19 @@ __global__ __launch_bounds__(1024) void tiny_kernel(ChebArgs<R> a, int F, int fi
             }
             if (p + 1 < (1 << F)) prefetch(j + 1);
         } else {
-            for (int t = 0; t < a.ncoef; ++t) {
-                const C c = j < a.N ? slice_coefficient(a.ctl, t, a.j0 + (int)j) : mk<R>(0, 0);
-                each([&](int k) {
-                    if (in[k]) x[k] = cadd(x[k], cmul(c, ops[t * dd + at[k]]));
-                });
+            for (int t0 = 0; t0 < a.ncoef; t0 += PER) {
+                wave_order();
+                cf[lane] = ahead;
+                wave_order();
+                const bool more = t0 + PER < a.ncoef;
+                ahead = evaluate(more ? t0 + PER + mine : mine, more ? p : p + 1);
+                const int cnt = min(PER, a.ncoef - t0);
+                for (int t = 0; t < cnt; ++t) {
+                    const C c = cf[L.q * PER + t];
+                    each([&](int k) {
+                        if (in[k]) x[k] = cadd(x[k], cmul(c, ops[(t0 + t) * dd + at[k]]));
+                    });
+                }
             }
         }
         if constexpr (SCHEME == 0) {
@@ -347,7 +369,7 @@ template <class R> hipError_t launch_tiny(const ChebArgs<R>& a, hipStream_t st) 
     const TinyPlan p = tiny_plan<R>(a.N, a.d);
     const int nc = a.ncoef <= 3 ? a.ncoef : 0;
     auto go = [&](auto kern, int ns, int sl) {
-        const size_t lds = ((size_t)p.waves * 2 * ns * sl + (nc ? 0 : (size_t)a.ncoef * a.d * a.d)) * sizeof(cplx<R>);
+        const size_t lds = ((size_t)p.waves * 2 * ns * sl + (nc ? 0 : (size_t)a.ncoef * a.d * a.d + 64 * p.waves)) * sizeof(cplx<R>);
         hipLaunchKernelGGL(kern, dim3(p.nodes), dim3(64 * p.waves), lds, st, a, p.fold, p.nodes == 1 ? 1 : 0);
     };
 #define PA_TINY(BD, SC)                                                                     \

@@ -239,3 +239,27 @@ def test_complex64_gradient_keeps_the_power_form(d, n):
             res.append(p.gate_fidelity_gradient(dt, *c, target=t))
             assert p.iteration_cycles == 9
     assert res[0][0] == res[1][0] and np.array_equal(res[0][1], res[1][1])
+
+
+@pytest.mark.parametrize("prec, d, amps, n", [("fp32", 3, 4, 50), ("fp32", 4, 7, 4097), ("fp32", 8, 16, 65), ("fp32", 8, 64, 20000),
+                                              ("fp32", 5, 17, 1), ("fp64", 4, 16, 129), ("fp64", 2, 33, 300), ("fp64", 8, 64, 1030),
+                                              ("fp64", 7, 20, 17)])
+@pytest.mark.parametrize("mode", ["none", "midpoint", "magnus"])
+def test_small_dims_many_operators(prec, d, amps, n, mode):
+    """Dims up to 8 with more operators than registers hold: coefficients dealt to the lanes in full and
+    partial rounds, at up to 64 of them (Magnus: as many controls as stay within 64 terms)."""
+    import parament_amd as parament
+    from tests.helpers import as_c64_inputs
+    if mode == "magnus":
+        amps = min(amps, 9)   # 9 + 9 + 36 terms
+    pts = 2 * n + 1 if mode == "magnus" else n + (mode == "midpoint")
+    h0, hks, c, dt = problem(d, amps, pts, 0.1, mode == "magnus")
+    quad = "simpson" if mode == "magnus" else mode
+    with parament.Parament(prec) as p:
+        p.set_hamiltonian(h0, *hks, quadrature_mode=quad, use_magnus=mode == "magnus")
+        u = p.equiprop(dt, *c)
+        m = p.iteration_cycles
+    if prec == "fp32":
+        h0, hks, c = as_c64_inputs(h0, hks, c)
+    ref = eo.equiprop(h0, hks, c, dt, mode=quad, use_magnus=mode == "magnus", cycles=m)
+    assert rel_err(u, ref) < (1e-12 if prec == "fp64" else 1e-5 + 2.0 ** -23 * n * 0.1)
