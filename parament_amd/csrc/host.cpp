@@ -333,7 +333,9 @@ template <class R> struct Context {
     void* d_nodes = nullptr; size_t cap_nodes = 0;
     pa::BufferSet gen;   // step-wise working arrays
     void* d_root = nullptr; size_t cap_root = 0;  // d x d result of the last equiprop
-    char* pin = nullptr; bool pin_failed = false; // host-array calls: pinned controls, then the result (kPin*)
+    // host-array calls: pin_in bytes of pinned controls, then pin_out of the result (kPin*)
+    char* pin = nullptr; size_t pin_in = 0, pin_out = 0;
+    bool pin_failed = false;
     void* d_c64 = nullptr; size_t cap_c64 = 0;    // complex64 contexts: controls widened to FP64
     void* d_out64 = nullptr; size_t cap_out64 = 0;  // complex64 contexts: FP64 result before rounding
     // gradient: leaves E, tree levels V, costates W, per-slice traces, trace g; tree layout policy
@@ -370,7 +372,7 @@ template <class R> void free_working(Context<R>* h) {
     hipFree(h->d_nodes); h->d_nodes = nullptr; h->cap_nodes = 0;
     h->gen.clear([](void* p) { hipFree(p); });
     hipFree(h->d_root); h->d_root = nullptr; h->cap_root = 0;
-    if (h->pin) { hipHostFree(h->pin); h->pin = nullptr; }
+    if (h->pin) { hipHostFree(h->pin); h->pin = nullptr; h->pin_in = h->pin_out = 0; }
     hipFree(h->d_c64); h->d_c64 = nullptr; h->cap_c64 = 0;
     hipFree(h->d_out64); h->d_out64 = nullptr; h->cap_out64 = 0;
     for (void** p : {&h->d_gE, &h->d_gV, &h->d_gW, &h->d_gdg, &h->d_gaux}) { hipFree(*p); *p = nullptr; }
@@ -1149,21 +1151,24 @@ Parament_ErrorCode run(Context<R>* h, const cplx<R>* carr_dev, double dt, unsign
         }
         const int F = small ? pa::small_fold_levels(N) : 0;
         const int n_nodes = tiny ? pa::tiny_nodes<R>(N, (int)d) : (N + (1 << F) - 1) >> F;
+        if (tiny && n_nodes == 1) {   // the launch reduces all slices and writes U itself
+            ca.out = out_dev;
+            mark(h, 0);
+            if (pa::launch_tiny<R>(ca, st) != hipSuccess) return PARAMENT_STATUS_CUBLAS_FAILED;
+            mark(h, 1);
+            mark(h, 2);
+            return PARAMENT_STATUS_SUCCESS;
+        }
         const size_t nodes = (size_t)pa::tree_scratch_nodes<R>(n_nodes);
         void* leaves = ws.get(&h->d_leaves, &h->cap_leaves, (size_t)n_nodes * dd * sizeof(C));
         void* scratch_nodes = leaves ? ws.get(&h->d_nodes, &h->cap_nodes, 2 * nodes * dd * sizeof(C)) : nullptr;
         if (!scratch_nodes) return ws.failure();
-        const bool whole = tiny && n_nodes == 1;   // the launch reduces all slices: it writes U itself
-        ca.out = whole ? out_dev : reinterpret_cast<C*>(leaves);
+        ca.out = reinterpret_cast<C*>(leaves);
         mark(h, 0);
         if ((tiny ? pa::launch_tiny<R>(ca, st) : small ? pa::launch_small_fold<R>(ca, st) : pa::launch_cheb_fused<R>(ca, st)) !=
             hipSuccess)
             return PARAMENT_STATUS_CUBLAS_FAILED;
         mark(h, 1);
-        if (whole) {
-            mark(h, 2);
-            return PARAMENT_STATUS_SUCCESS;
-        }
         C* nd = reinterpret_cast<C*>(scratch_nodes);
         if (pa::launch_tree<R>(leaves, false, n_nodes, (int)d, nd, nd + nodes * dd, out_dev, st) != hipSuccess)
             return PARAMENT_STATUS_CUBLAS_FAILED;
@@ -1301,22 +1306,35 @@ template <class R> Parament_ErrorCode ensure_common(Context<R>* h, unsigned amps
 
 // Host-array calls stage controls of up to kPinIn bytes and results of up to kPinOut in pinned memory, which the
 // kernels read and write across the bus: a copy of either to or from the caller's pageable array takes 8 to 12 us,
-// more than a small problem's launches.  Controls up to kPinDirect are read where they are by a one-launch
+// more than a small problem's launches.  It is allocated as large as the arrays need (grow-only): 4 KB take 26 us, all of
+// it 42, in a context's first call.  Controls up to kPinDirect are read where they are by a one-launch
 // problem (each sample once); larger ones go to the device by a kernel.  Larger arrays take copies, whose
 // rate is then what counts.
 constexpr size_t kPinIn = 512 << 10, kPinOut = 64 << 10, kPinDirect = 4 << 10;
 
-template <class R> bool pinned(Context<R>* h) {
-    if (!h->pin && !h->pin_failed) {
-        void* p = nullptr;
-        if (hipHostMalloc(&p, kPinIn + kPinOut) != hipSuccess) {
-            hipGetLastError();
-            h->pin_failed = true;
-        } else {
-            h->pin = static_cast<char*>(p);
-        }
+// Whether pinned memory holds controls of in bytes and a result of out bytes (0: not staged).
+template <class R> bool pinned(Context<R>* h, size_t in, size_t out) {
+    if (h->pin_in >= in && h->pin_out >= out) return true;
+    if (h->pin_failed) return false;
+    auto room = [](size_t need, size_t held) {   // doubling, so that growing lengths allocate seldom
+        size_t b = std::max<size_t>(held, 2048);
+        while (b < need) b *= 2;
+        return b;
+    };
+    const size_t b_in = room(in, h->pin_in), b_out = room(out, h->pin_out);
+    if (h->pin) hipHostFree(h->pin);
+    h->pin = nullptr;
+    h->pin_in = h->pin_out = 0;
+    void* p = nullptr;
+    if (hipHostMalloc(&p, b_in + b_out) != hipSuccess) {
+        hipGetLastError();
+        h->pin_failed = true;
+        return false;
     }
-    return h->pin != nullptr;
+    h->pin = static_cast<char*>(p);
+    h->pin_in = b_in;
+    h->pin_out = b_out;
+    return true;
 }
 
 template <class R>
@@ -1330,7 +1348,9 @@ Parament_ErrorCode equiprop(Context<R>* h, const typename ApiCplx<R>::type* carr
     if (err != PARAMENT_STATUS_SUCCESS) return h->last_error = err;
     const size_t dd = (size_t)h->dim * h->dim;
     const size_t cbytes = (size_t)amps * pts * sizeof(C);
-    const bool pin_in = cbytes <= kPinIn && pinned(h), pin_out = dd * sizeof(C) <= kPinOut && pinned(h);
+    const bool in_fits = cbytes <= kPinIn, out_fits = dd * sizeof(C) <= kPinOut;
+    const bool staged = (in_fits || out_fits) && pinned(h, in_fits ? cbytes : 0, out_fits ? dd * sizeof(C) : 0);
+    const bool pin_in = staged && in_fits, pin_out = staged && out_fits;
     const bool direct = pin_in && cbytes <= kPinDirect && h->path == 0 && !uses_mixed(h) && pa::tiny_supported((int)h->dim, h->ncoef);
     if (!direct && !grow(reinterpret_cast<void**>(&h->d_c), &h->cap_c, std::max<size_t>(cbytes, sizeof(C))))
         return h->last_error = PARAMENT_STATUS_DEVICE_ALLOC_FAILED;
@@ -1338,7 +1358,7 @@ Parament_ErrorCode equiprop(Context<R>* h, const typename ApiCplx<R>::type* carr
     if (!direct && (pin_in ? pa::launch_stage(h->pin, cbytes, h->d_c, h->stream)
                            : hipMemcpyAsync(h->d_c, carr, cbytes, hipMemcpyHostToDevice, h->stream)) != hipSuccess)
         return h->last_error = PARAMENT_STATUS_CUBLAS_FAILED;
-    C* root = pin_out ? reinterpret_cast<C*>(h->pin + kPinIn) : reinterpret_cast<C*>(h->d_root);
+    C* root = pin_out ? reinterpret_cast<C*>(h->pin + h->pin_in) : reinterpret_cast<C*>(h->d_root);
     err = run_replayable(h, direct ? reinterpret_cast<const C*>(h->pin) : h->d_c, dt, pts, amps, root);
     if (err == PARAMENT_STATUS_SUCCESS) {
         if ((!pin_out && hipMemcpyAsync(out, root, dd * sizeof(C), hipMemcpyDeviceToHost, h->stream) != hipSuccess) ||

@@ -263,3 +263,25 @@ def test_small_dims_many_operators(prec, d, amps, n, mode):
         h0, hks, c = as_c64_inputs(h0, hks, c)
     ref = eo.equiprop(h0, hks, c, dt, mode=quad, use_magnus=mode == "magnus", cycles=m)
     assert rel_err(u, ref) < (1e-12 if prec == "fp64" else 1e-5 + 2.0 ** -23 * n * 0.1)
+
+
+@pytest.mark.parametrize("prec, d", [("fp32", 2), ("fp64", 8), ("fp64", 40)])
+def test_host_arrays_of_changing_length(prec, d):
+    """One context over host arrays that grow and shrink, within the pinned memory's sizes, past their
+    doublings and beyond them: each call the device-array call's bits."""
+    import torch
+    import parament_amd as parament
+    ct, rt = (torch.complex64, np.complex64) if prec == "fp32" else (torch.complex128, np.complex128)
+    h0, hks, c, dt = problem(d, 2, 40000, 0.02, False)
+    c = c.astype(rt)
+    with parament.Parament(prec) as p:
+        p.set_hamiltonian(h0, *hks)
+        for n in (5, 64, 65, 3, 1000, 1000, 1000, 20000, 7, 40000, 300):
+            block = np.ascontiguousarray(c[:, n // 3:n // 3 + n] if n < 20000 else c[:, :n])
+            u = p.equiprop(dt, *block)
+            carr = torch.tensor(block, dtype=ct, device="cuda")
+            out = torch.empty((d, d), dtype=ct, device="cuda")
+            torch.cuda.synchronize()
+            p.equiprop_device(dt, carr.data_ptr(), n, 2, out.data_ptr())
+            p.synchronize()
+            assert np.array_equal(u, out.cpu().numpy()), n
