@@ -326,7 +326,7 @@ template <class R> struct Context {
     C* d_ops = nullptr;
     // complex64 contexts: the operators (Magnus commutators included) in FP64, for the mixed pipeline
     double2* d_ops64 = nullptr;
-    double2* d_opsP = nullptr;   // dims <= 64: the operators in FP64 padded for the fp16 split kernel
+    double2* d_opsP = nullptr;   // the operators in FP64 padded for the fp16 split kernel, where it is used
     // working memory (grow-only, like parament.cpp:418)
     C* d_c = nullptr; size_t cap_c = 0;
     void* d_leaves = nullptr; size_t cap_leaves = 0;
@@ -697,6 +697,27 @@ template <class R> hipError_t magnus_commutators(cplx<R>* ops, unsigned d, unsig
     return hipSuccess;
 }
 
+// The fp16 split kernel's padded operators, for contexts whose precision mode and dim use it (and not the
+// complex64 default mode's own kernels up to dim 16).  Without memory for them there are none, and run_mixed_fused
+// takes the bf16 split kernel, which reads the operators as they are.  True when work was enqueued on st.
+template <class R> bool pad_operators(Context<R>* h, hipStream_t st) {
+    const bool used = h->precision == PARAMENT_PRECISION_MIXED && pa::mixed_supported((int)h->dim) &&
+                      mixed_split_scheme() != 0 && !(sizeof(R) == 4 && h->dim <= 16);
+    if (!used || h->d_opsP) return false;
+    const int nops = 1 + h->ncoef;
+    const size_t pd = (size_t)pa::h2_padded_dim((int)h->dim);
+    const double2* src = sizeof(R) == 8 ? reinterpret_cast<const double2*>(h->d_ops) : h->d_ops64;
+    void* p = nullptr;
+    if (hipMalloc(&p, nops * pd * pd * sizeof(double2)) == hipSuccess &&
+        pa::launch_pad(src, nops, (int)h->dim, reinterpret_cast<double2*>(p), st) == hipSuccess) {
+        h->d_opsP = reinterpret_cast<double2*>(p);
+        return true;
+    }
+    hipGetLastError();
+    if (p) hipFree(p);
+    return false;
+}
+
 template <class R>
 Parament_ErrorCode set_hamiltonian(Context<R>* h, const typename ApiCplx<R>::type* H0, const typename ApiCplx<R>::type* H1,
                                    unsigned dim, unsigned amps, bool use_magnus, int quad) {
@@ -761,20 +782,7 @@ Parament_ErrorCode set_hamiltonian(Context<R>* h, const typename ApiCplx<R>::typ
         free_hamiltonian(h);
         return h->last_error = PARAMENT_STATUS_CUBLAS_FAILED;
     }
-    if (pa::mixed_supported((int)dim)) {
-        const size_t pd = (size_t)pa::h2_padded_dim((int)dim);
-        if (hipMalloc(&h->d_opsP, nops * pd * pd * sizeof(double2)) != hipSuccess) {
-            hipGetLastError();
-            h->d_opsP = nullptr;
-            free_hamiltonian(h);
-            return h->last_error = PARAMENT_STATUS_DEVICE_ALLOC_FAILED;
-        }
-        const double2* src = sizeof(R) == 8 ? reinterpret_cast<const double2*>(h->d_ops) : h->d_ops64;
-        if (pa::launch_pad(src, (int)nops, (int)dim, h->d_opsP, h->stream) != hipSuccess) {
-            free_hamiltonian(h);
-            return h->last_error = PARAMENT_STATUS_CUBLAS_FAILED;
-        }
-    }
+    pad_operators(h, h->stream);
     if (hipStreamSynchronize(h->stream) != hipSuccess) {
         free_hamiltonian(h);
         return h->last_error = PARAMENT_STATUS_CUBLAS_FAILED;
@@ -1041,7 +1049,7 @@ Parament_ErrorCode run_mixed_fused(Context<R>* h, const MixedSrc& m, double2* ou
     void* scratch_nodes = leaves ? ws.get(&h->d_nodes, &h->cap_nodes, 2 * nodes * dd * sizeof(double2)) : nullptr;
     if (!scratch_nodes) return ws.failure();
     ma.out = reinterpret_cast<float2*>(leaves);
-    const int split = mixed_split_scheme();
+    const int split = h->d_opsP ? mixed_split_scheme() : 0;
     if (ma.ps && split) {
         ma.ops = h->d_opsP;
         h2_coefficients(ma, M, xarg, h->manual);
@@ -1992,6 +2000,13 @@ template <class R> Parament_ErrorCode set_precision(Context<R>* h, int mode) {
         mode != PARAMENT_PRECISION_MIXED_BF16X2)
         return h->last_error = PARAMENT_STATUS_INVALID_VALUE;
     h->precision = mode;
+    if (h->has_h && hipSetDevice(h->device) == hipSuccess) {
+        // a setter may be called while a stream of this thread is captured
+        hipStreamCaptureMode capture = hipStreamCaptureModeRelaxed;
+        hipThreadExchangeStreamCaptureMode(&capture);
+        if (pad_operators(h, h->own_stream)) hipStreamSynchronize(h->own_stream);
+        hipThreadExchangeStreamCaptureMode(&capture);
+    }
     return h->last_error = PARAMENT_STATUS_SUCCESS;
 }
 
