@@ -89,7 +89,7 @@ struct EpiIO {
 // + ca A + cb B + diag, and the second output's combination, in FP64, rounded once.  Each element
 // reads its own Cin / Cin2 positions before it is written, so C or D may be one of them.  A, B point
 // at product b's operands.
-// EP_GENERAL serves ca, cb and the second output; EP_PLAIN ca = cb = 0 or 1; EP_DUAL none of them.
+// EP_GENERAL (complex128) serves ca, cb and the second output; EP_PLAIN ca = cb = 0 or 1; EP_DUAL none of them.
 template <int EP, class TA, class TB, class TC, class TO>
 __device__ __forceinline__ void epi_store(const GemmArgs& g, const EpiIO<TA, TB, TC, TO>& io, const TA* A,
                                           const TB* B, long b, long dd, long o, bool on_diag, double xr, double xi) {
@@ -226,7 +226,7 @@ __global__ __launch_bounds__((fp_threads<R, BT>()), sizeof(R) == 8 ? 4 : 1) void
 // waves, wave w the 16-row band [16 w, 16 w + 16) over all 16 NW columns, so the padding is to a
 // multiple of 16 and every operand element is fetched once per product.  K in chunks of 32,
 // the next one fetched into registers while the matrix cores work on the current one.
-template <int NW, int EP, class TA, class TB, class TC, class TO>
+template <int NW, class TA, class TB, class TC, class TO>
 __global__ __launch_bounds__(64 * NW) void zgemm_row_kernel(GemmArgs g, EpiIO<TA, TB, TC, TO> io) {
     typedef float R;
     constexpr int DP = 16 * NW, NT = 64 * NW;
@@ -280,7 +280,7 @@ __global__ __launch_bounds__(64 * NW) void zgemm_row_kernel(GemmArgs g, EpiIO<TA
         for (int v = 0; v < 4; ++v) {
             const int gi = acc_row<R>(wr, 0, v), gj = acc_col(0, n);
             if (gi >= d || gj >= d) continue;
-            epi_store<EP>(g, io, A, B, b, dd, (long)gi * d + gj, gi == gj, acc.re[0][n][v], acc.im[0][n][v]);
+            epi_store<EP_PLAIN>(g, io, A, B, b, dd, (long)gi * d + gj, gi == gj, acc.re[0][n][v], acc.im[0][n][v]);
         }
 }
 
@@ -289,8 +289,7 @@ __global__ __launch_bounds__(64 * NW) void zgemm_row_kernel(GemmArgs g, EpiIO<TA
 // lane l holds A[l%16][8(l/16) .. +7] and Bt[l%16][8(l/16) .. +7]; accumulator element v is
 // C[4(l/16) + v][l%16].  F16: the scaled fp16 two-way split (NS = 2), else bf16 slices.  EDGE:
 // d is not a multiple of BT, so loads and stores past d are masked (otherwise none is).  EP: the launch
-// has a second product (EP_DUAL), a second output or ca, cb other than both 0 or both 1 (EP_GENERAL), or
-// neither (EP_PLAIN; kept apart because the general epilogue's registers cost the others 1-2%).
+// has a second product (EP_DUAL) or not (EP_PLAIN).
 template <int NS, int BT, bool F16, bool EDGE, int EP, class TA, class TB, class TC, class TO>
 __global__ __launch_bounds__(256) void zgemm_split_kernel(GemmArgs g, EpiIO<TA, TB, TC, TO> io) {
     constexpr bool DUAL = EP == EP_DUAL;
@@ -477,10 +476,7 @@ __global__ __launch_bounds__(256) void zgemm_split_kernel(GemmArgs g, EpiIO<TA, 
         const float b_re = (float)g.beta_re, b_im = (float)g.beta_im;
         const float c_re = (float)g.beta2_re, c_im = (float)g.beta2_im;
         const float g_re = (float)g.diag_re, g_im = (float)g.diag_im;
-        const float ga = (float)g.ca, gb = (float)g.cb;
-        const float dab = (float)(g.d_ab * kF16Unscale), da = (float)g.d_a, db = (float)g.d_b, dc = (float)g.d_c,
-                    dc2 = (float)g.d_c2;
-        const bool has_a = g.ca != 0.0 || g.d_a != 0.0, has_b = g.cb != 0.0 || g.d_b != 0.0;
+        const bool add_ab = EP == EP_PLAIN && g.ca != 0.0;
         const long ib = b * g.sc * dd, ib2 = b * g.sc2 * dd, ob = b * g.so * dd;
 #pragma unroll
         for (int m = 0; m < TW; ++m)
@@ -493,41 +489,25 @@ __global__ __launch_bounds__(256) void zgemm_split_kernel(GemmArgs g, EpiIO<TA, 
                     const long o = (long)gi * d + gj;
                     const float xr = accr[0][m][n][v], xi = acci[0][m][n][v];
                     float yr = a_re * xr - a_im * xi, yi = a_re * xi + a_im * xr;
-                    float zr = dab * xr, zi = dab * xi;
                     if (io.Cin) {
                         const TC cv = io.Cin[ib + o];
                         yr = __builtin_fmaf(b_re, cv.x, __builtin_fmaf(-b_im, cv.y, yr));
                         yi = __builtin_fmaf(b_re, cv.y, __builtin_fmaf(b_im, cv.x, yi));
-                        zr = __builtin_fmaf(dc, cv.x, zr); zi = __builtin_fmaf(dc, cv.y, zi);
                     }
                     if (io.Cin2) {
                         const TC cv = io.Cin2[ib2 + o];
                         yr = __builtin_fmaf(c_re, cv.x, __builtin_fmaf(-c_im, cv.y, yr));
                         yi = __builtin_fmaf(c_re, cv.y, __builtin_fmaf(c_im, cv.x, yi));
-                        zr = __builtin_fmaf(dc2, cv.x, zr); zi = __builtin_fmaf(dc2, cv.y, zi);
                     }
-                    if (EP == EP_PLAIN && has_a) {
+                    if (add_ab) {
                         const TA av = A[o];
                         const TB bv = B[o];
                         yr += av.x + bv.x; yi += av.y + bv.y;
-                    }
-                    if (EP == EP_GENERAL) {
-                        TA av;
-                        TB bv;
-                        av.x = av.y = 0; bv.x = bv.y = 0;
-                        if (has_a) av = A[o];
-                        if (has_b) bv = B[o];
-                        yr += __builtin_fmaf(ga, av.x, gb * bv.x); yi += __builtin_fmaf(ga, av.y, gb * bv.y);
-                        zr += __builtin_fmaf(da, av.x, db * bv.x); zi += __builtin_fmaf(da, av.y, db * bv.y);
                     }
                     if (gi == gj) { yr += g_re; yi += g_im; }
                     TO out;
                     out.x = yr; out.y = yi;
                     io.C[ob + o] = out;
-                    if (EP == EP_GENERAL && io.D) {
-                        out.x = zr; out.y = zi;
-                        io.D[ob + o] = out;
-                    }
                 }
         return;
     }
@@ -559,9 +539,8 @@ __global__ __launch_bounds__(256) void zgemm_split_kernel(GemmArgs g, EpiIO<TA, 
 // the compiler from moving loads over stores): one at a time they cost 4 ms of the 11.1 ms that 16,384
 // dim-256 products with two inputs took with 64x64 tiles.  A product without inputs takes 361 ns at dim 256, of
 // which the matrix cores' own work is 160 and the split and the epilogue, which overlap it in part, 75 and 65.
-template <bool EDGE, int EP>
+template <bool EDGE, bool DUAL>
 __global__ __launch_bounds__(512, 2) void zgemm_f16_kernel(GemmArgs g, EpiIO<float2, float2, float2, float2> io) {
-    constexpr bool DUAL = EP == EP_DUAL;
     constexpr int BT = 128, TM = 4, TN = 2, PL = BT * KT;
     typedef _Float16 f16x4g __attribute__((ext_vector_type(4)));
     typedef float f32x4u __attribute__((ext_vector_type(4), aligned(8)));
@@ -706,10 +685,7 @@ __global__ __launch_bounds__(512, 2) void zgemm_f16_kernel(GemmArgs g, EpiIO<flo
     const float b_re = (float)g.beta_re, b_im = (float)g.beta_im;
     const float c_re = (float)g.beta2_re, c_im = (float)g.beta2_im;
     const float g_re = (float)g.diag_re, g_im = (float)g.diag_im;
-    const float ca = (float)g.ca, cb = (float)g.cb;
-    const float dab = (float)(g.d_ab * kF16Unscale), da = (float)g.d_a, db = (float)g.d_b, dc = (float)g.d_c,
-                dc2 = (float)g.d_c2;
-    const bool has_a = !DUAL && (g.ca != 0.0 || g.d_a != 0.0), has_b = !DUAL && (g.cb != 0.0 || g.d_b != 0.0);
+    const bool add_ab = !DUAL && g.ca != 0.0;
     auto epilogue = [&](long item) {
         const long b = item / tt;
         const int t = (int)(item % tt), i0 = (t / tiles) * BT, j0 = (t % tiles) * BT;
@@ -718,7 +694,6 @@ __global__ __launch_bounds__(512, 2) void zgemm_f16_kernel(GemmArgs g, EpiIO<flo
         const float2* Cin = io.Cin ? io.Cin + b * g.sc * dd : nullptr;
         const float2* Cin2 = io.Cin2 ? io.Cin2 + b * g.sc2 * dd : nullptr;
         float2* C = io.C + b * g.so * dd;
-        float2* D2 = EP == EP_GENERAL && io.D ? io.D + b * g.so * dd : nullptr;
         struct In { float2 c[4], c2[4], a[4], b[4]; };
         auto at = [&](int blk, int v) -> unsigned {
             const int gi = i0 + wr + 16 * (blk / TN) + 4 * kq + v, gj = j0 + wc + 16 * (blk % TN) + r16;
@@ -730,8 +705,7 @@ __global__ __launch_bounds__(512, 2) void zgemm_f16_kernel(GemmArgs g, EpiIO<flo
                 const unsigned o = at(blk, v);
                 if (Cin) x.c[v] = Cin[o];
                 if (Cin2) x.c2[v] = Cin2[o];
-                if (has_a) x.a[v] = A[o];
-                if (has_b) x.b[v] = B[o];
+                if (add_ab) { x.a[v] = A[o]; x.b[v] = B[o]; }
             }
         };
         In cur, nxt;
@@ -747,35 +721,21 @@ __global__ __launch_bounds__(512, 2) void zgemm_f16_kernel(GemmArgs g, EpiIO<flo
                 const unsigned o = (unsigned)gi * d + gj;
                 const float xr = accr[m][n][v], xi = acci[m][n][v];
                 float yr = a_re * xr - a_im * xi, yi = a_re * xi + a_im * xr;
-                float zr = dab * xr, zi = dab * xi;
                 if (Cin) {
                     const float2 c = cur.c[v];
                     yr = __builtin_fmaf(b_re, c.x, __builtin_fmaf(-b_im, c.y, yr));
                     yi = __builtin_fmaf(b_re, c.y, __builtin_fmaf(b_im, c.x, yi));
-                    zr = __builtin_fmaf(dc, c.x, zr); zi = __builtin_fmaf(dc, c.y, zi);
                 }
                 if (Cin2) {
                     const float2 c = cur.c2[v];
                     yr = __builtin_fmaf(c_re, c.x, __builtin_fmaf(-c_im, c.y, yr));
                     yi = __builtin_fmaf(c_re, c.y, __builtin_fmaf(c_im, c.x, yi));
-                    zr = __builtin_fmaf(dc2, c.x, zr); zi = __builtin_fmaf(dc2, c.y, zi);
                 }
-                if (EP == EP_PLAIN && has_a) {
+                if (add_ab) {
                     yr += cur.a[v].x + cur.b[v].x; yi += cur.a[v].y + cur.b[v].y;
-                }
-                if (EP == EP_GENERAL) {
-                    if (has_a) {
-                        yr = __builtin_fmaf(ca, cur.a[v].x, yr); yi = __builtin_fmaf(ca, cur.a[v].y, yi);
-                        zr = __builtin_fmaf(da, cur.a[v].x, zr); zi = __builtin_fmaf(da, cur.a[v].y, zi);
-                    }
-                    if (has_b) {
-                        yr = __builtin_fmaf(cb, cur.b[v].x, yr); yi = __builtin_fmaf(cb, cur.b[v].y, yi);
-                        zr = __builtin_fmaf(db, cur.b[v].x, zr); zi = __builtin_fmaf(db, cur.b[v].y, zi);
-                    }
                 }
                 if (gi == gj) { yr += g_re; yi += g_im; }
                 C[o] = make_float2(yr, yi);
-                if (EP == EP_GENERAL && D2) D2[o] = make_float2(zr, zi);
             }
             cur = nxt;
         }
@@ -823,15 +783,10 @@ hipError_t launch_f16(const GemmArgs& g, const EpiIO<float2, float2, float2, flo
     // persistent: one work-group per CU (its LDS), each looping over output tiles with the next tile's first
     // chunks fetched before the epilogue
     const dim3 grid((unsigned)std::min<long>(total, 256)), block(512);
-    const int ep = epilogue(g);
-#define PA_F16(E)                                                                                \
-    if (g.d % 128) hipLaunchKernelGGL((zgemm_f16_kernel<true, E>), grid, block, 0, st, g, io);   \
-    else hipLaunchKernelGGL((zgemm_f16_kernel<false, E>), grid, block, 0, st, g, io);
-    switch (ep) {
-        case EP_DUAL: PA_F16(EP_DUAL) break;
-        case EP_PLAIN: PA_F16(EP_PLAIN) break;
-        default: PA_F16(EP_GENERAL) break;
-    }
+#define PA_F16(DU)                                                                                \
+    if (g.d % 128) hipLaunchKernelGGL((zgemm_f16_kernel<true, DU>), grid, block, 0, st, g, io);   \
+    else hipLaunchKernelGGL((zgemm_f16_kernel<false, DU>), grid, block, 0, st, g, io);
+    if (g.A2) { PA_F16(true) } else { PA_F16(false) }
 #undef PA_F16
     return hipGetLastError();
 }
@@ -848,11 +803,14 @@ hipError_t launch_tiled(const GemmArgs& g, int mode, const EpiIO<TA, TB, TC, TO>
 #define PA_FP2(R, DU)                                                                                                   \
     if (g.d % BT) hipLaunchKernelGGL((zgemm_fp_kernel<R, BT, true, DU, TA, TB, TC, TO>), grid, dim3(fp_threads<R, BT>()), 0, st, g, io);   \
     else hipLaunchKernelGGL((zgemm_fp_kernel<R, BT, false, DU, TA, TB, TC, TO>), grid, dim3(fp_threads<R, BT>()), 0, st, g, io);
-#define PA_FP(R) if (ep == EP_DUAL) { PA_FP2(R, EP_DUAL) } else if (ep == EP_PLAIN) { PA_FP2(R, EP_PLAIN) } \
-    else { PA_FP2(R, EP_GENERAL) }
-        case GEMM_F64: PA_FP(double) break;
-        case GEMM_F32: PA_FP(float) break;
-#undef PA_FP
+        case GEMM_F64:
+            if constexpr (sizeof(TA) == 16)
+                if (ep == EP_GENERAL) { PA_FP2(double, EP_GENERAL) break; }
+            if (ep == EP_DUAL) { PA_FP2(double, EP_DUAL) } else { PA_FP2(double, EP_PLAIN) }
+            break;
+        case GEMM_F32:
+            if (ep == EP_DUAL) { PA_FP2(float, EP_DUAL) } else { PA_FP2(float, EP_PLAIN) }
+            break;
 #undef PA_FP2
 #define PA_SPLIT(NS, F16, DU)                                                                                          \
     if (g.d % BT) hipLaunchKernelGGL((zgemm_split_kernel<NS, BT, F16, true, DU, TA, TB, TC, TO>), grid, block, 0, st, g, io); \
@@ -860,9 +818,7 @@ hipError_t launch_tiled(const GemmArgs& g, int mode, const EpiIO<TA, TB, TC, TO>
         case GEMM_BF16X2: PA_SPLIT(2, false, EP_PLAIN) break;
         case GEMM_BF16X3: PA_SPLIT(3, false, EP_PLAIN) break;
         case GEMM_F16X2:
-            if (ep == EP_DUAL) { PA_SPLIT(2, true, EP_DUAL) }
-            else if (ep == EP_PLAIN) { PA_SPLIT(2, true, EP_PLAIN) }
-            else { PA_SPLIT(2, true, EP_GENERAL) }
+            if (ep == EP_DUAL) { PA_SPLIT(2, true, EP_DUAL) } else { PA_SPLIT(2, true, EP_PLAIN) }
             break;
 #undef PA_SPLIT
         default: return hipErrorInvalidValue;
@@ -875,10 +831,7 @@ hipError_t launch_row(const GemmArgs& g, const EpiIO<TA, TB, TC, TO>& io, hipStr
     const int nw = (g.d + 15) / 16;
     if (g.batch <= 0) return hipSuccess;
     const dim3 grid((unsigned)g.batch);
-    const bool general = epilogue(g) == EP_GENERAL;
-#define PA_ROW(NW)                                                                                                      \
-    if (general) hipLaunchKernelGGL((zgemm_row_kernel<NW, EP_GENERAL, TA, TB, TC, TO>), grid, dim3(64 * NW), 0, st, g, io); \
-    else hipLaunchKernelGGL((zgemm_row_kernel<NW, EP_PLAIN, TA, TB, TC, TO>), grid, dim3(64 * NW), 0, st, g, io);
+#define PA_ROW(NW) hipLaunchKernelGGL((zgemm_row_kernel<NW, TA, TB, TC, TO>), grid, dim3(64 * NW), 0, st, g, io);
     switch (nw) {
         case 3: PA_ROW(3) break;
         case 4: PA_ROW(4) break;
@@ -921,6 +874,8 @@ hipError_t launch_zgemm(const GemmArgs& g, int mode, hipStream_t st) {
     if ((g.A2 || g.B2) &&
         (!g.A2 || !g.B2 || mode == GEMM_BF16X2 || mode == GEMM_BF16X3 || g.ca != 0.0 || g.cb != 0.0 || g.D))
         return hipErrorInvalidValue;
+    // a second output, or ca and cb other than both 0 or both 1: complex128 only
+    if (epilogue(g) == EP_GENERAL && !(mode == GEMM_F64 && g.a_c128 && g.b_c128)) return hipErrorInvalidValue;
     if (mode == GEMM_F64) {
         if (!g.out_c128) return hipErrorInvalidValue;
         if (g.a_c128 && g.b_c128) return launch_typed<double2, double2, double2, double2>(g, mode, st);

@@ -821,13 +821,13 @@ hipError_t launch_grad_slices(const ChebArgs<R>& a, const cplx<R>* E, const cplx
         return hipErrorInvalidValue;
     // the direct gradient needs one sample per slice and the traces of plain controls
     if (gd.grad && (a.ctl.mode != QUAD_NONE || a.ctl.magnus || !gd.g || gd.amps > a.ncoef)) return hipErrorInvalidValue;
-    if (a.pdeg && a.pdeg != 8 && a.pdeg != 12) return hipErrorInvalidValue;
+    if (a.pdeg && a.pdeg != 8 && (sizeof(R) == 4 || a.pdeg != 12)) return hipErrorInvalidValue;
     const dim3 grid(a.N);
 #define PA_GRAD_SLICES(DD)                                                                                              \
     {                                                                                                                   \
         const dim3 block(64 * Shape<DD>::G);                                                                            \
         if (a.pdeg == 8) hipLaunchKernelGGL((grad_slice_kernel<R, DD, 8>), grid, block, 0, st, a, E, W1, dg, dg_stride, gd); \
-        else if (a.pdeg) hipLaunchKernelGGL((grad_slice_kernel<R, DD, 12>), grid, block, 0, st, a, E, W1, dg, dg_stride, gd); \
+        else if (a.pdeg) hipLaunchKernelGGL((grad_slice_kernel<R, DD, sizeof(R) == 8 ? 12 : 8>), grid, block, 0, st, a, E, W1, dg, dg_stride, gd); \
         else if (a.ps) hipLaunchKernelGGL((grad_slice_kernel<R, DD, 1>), grid, block, 0, st, a, E, W1, dg, dg_stride, gd); \
         else hipLaunchKernelGGL((grad_slice_kernel<R, DD, 0>), grid, block, 0, st, a, E, W1, dg, dg_stride, gd);         \
     }

@@ -562,33 +562,29 @@ template <class R> PolyScheme stepwise_scheme(int M, double x, bool manual) {
 }
 inline int poly_buffers(const PolyScheme& p) { return p.deg == 12 ? 5 : 4; }
 
-// Slices E_j = p(X_j) - I of a batch of cnt slices on the schemes of poly_scheme, batched GEMMs, from
+// complex128 slices E_j = p(X_j) - I of a batch of cnt slices on the schemes of poly_scheme, batched GEMMs, from
 // Z = -i tau X (overwritten).  The operands that combine several matrices are second outputs of the GEMM
 // before, and the terms of the last step are written in the matrices it reads anyway:
 //   degree 8:  Z2 = Z Z,  L = Z + q3 Z2;  [P = Z2 L]  u = Z2 + q4 P,  a = Z + q5 Z2 + q6 P;
 //              E = q0 I + q8 u a + q1 a + y u + v Z2;
 //   degree 12: Z2 = Z Z;  Z3 = Z Z2,  B = Z + q4 Z2 + q5 Z3;  [P = B B]  u = P + q6 Z + q7 Z2 + q8 Z3,
 //              a = Z + q9 Z2 + q10 Z3 + q11 P  (Z = B - q4 Z2 - q5 Z3);  E = q0 I + q13 u a + t a + y u + v Z2 + v' Z3.
-// With first_order false the last step leaves out q1 Z + q0 I, which the caller adds (degree 8).
-// w: poly_buffers(p) - 1 buffers of cnt slices.  E goes to out, or, when out is null, to one of w
-// (*result says which); Z is free afterwards.
-template <class R>
-hipError_t poly_batched(int mode, const PolyScheme& p, cplx<R>* Z, int d, int cnt, bool first_order, cplx<R>* const* w,
-                        cplx<R>* out, cplx<R>** result, hipStream_t st, int tile = 0) {
+// w: poly_buffers(p) - 1 buffers of cnt slices, one of which receives E (*result says which); Z is free afterwards.
+hipError_t poly_batched(const PolyScheme& p, double2* Z, int d, int cnt, double2* const* w, double2** result, hipStream_t st) {
     const double* q = p.q;
     pa::GemmArgs g0;
-    g0.d = d; g0.batch = cnt; g0.tile = tile;
-    g0.a_c128 = g0.b_c128 = g0.out_c128 = sizeof(R) == 8;
+    g0.d = d; g0.batch = cnt;
+    g0.a_c128 = g0.b_c128 = g0.out_c128 = 1;
     g0.sa = g0.sb = g0.sc = g0.sc2 = g0.so = 1;
     g0.Cin = nullptr;
     g0.alpha_im = g0.beta_re = g0.beta_im = g0.diag_re = g0.diag_im = 0.0;
     g0.alpha_re = 1.0;
-    auto go = [&](pa::GemmArgs& g, const cplx<R>* A, const cplx<R>* B, cplx<R>* C) {
+    auto go = [&](pa::GemmArgs& g, const double2* A, const double2* B, double2* C) {
         g.A = A; g.B = B; g.C = C;
-        return pa::launch_zgemm(g, mode, st);
+        return pa::launch_zgemm(g, pa::GEMM_F64, st);
     };
     if (p.deg == 8) {
-        cplx<R>*Z2 = w[0], *L = w[1], *u = w[2], *a = Z;
+        double2*Z2 = w[0], *L = w[1], *u = w[2], *a = Z;
         pa::GemmArgs g = g0;
         g.Cin = Z; g.D = L; g.d_c = 1.0; g.d_ab = q[3];
         hipError_t r = go(g, Z, Z, Z2);
@@ -598,17 +594,16 @@ hipError_t poly_batched(int mode, const PolyScheme& p, cplx<R>* Z, int d, int cn
         if (r == hipSuccess) r = go(g, Z2, L, u);
         g = g0;
         // q1 Z + q2 Z2 + q7 P with P = (u - Z2) / q4 and Z = a - q5 Z2 - q6 P
-        const double t = first_order ? q[1] : 0.0, y = (q[7] - t * q[6]) / q[4];
+        const double t = q[1], y = (q[7] - t * q[6]) / q[4];
         g.alpha_re = q[8]; g.ca = y; g.cb = t;
         g.Cin = Z2; g.beta_re = q[2] - t * q[5] - y;
-        if (first_order) g.diag_re = q[0];
-        cplx<R>* E = out ? out : Z2;
-        if (r == hipSuccess) r = go(g, u, a, E);
-        if (result) *result = E;
+        g.diag_re = q[0];
+        if (r == hipSuccess) r = go(g, u, a, Z2);
+        *result = Z2;
         return r;
     }
-    if (p.deg != 12 || !first_order) return hipErrorInvalidValue;
-    cplx<R>*Z2 = w[0], *Z3 = w[1], *B = w[2], *u = w[3], *a = Z;
+    if (p.deg != 12) return hipErrorInvalidValue;
+    double2*Z2 = w[0], *Z3 = w[1], *B = w[2], *u = w[3], *a = Z;
     pa::GemmArgs g = g0;
     hipError_t r = go(g, Z, Z, Z2);
     g = g0;
@@ -625,9 +620,8 @@ hipError_t poly_batched(int mode, const PolyScheme& p, cplx<R>* Z, int d, int cn
     g.Cin = Z2; g.beta_re = q[2] - t * q[9] - y * q[7];
     g.Cin2 = Z3; g.beta2_re = q[3] - t * q[10] - y * q[8];
     g.diag_re = q[0];
-    cplx<R>* E = out ? out : Z3;
-    if (r == hipSuccess) r = go(g, u, a, E);
-    if (result) *result = E;
+    if (r == hipSuccess) r = go(g, u, a, Z3);
+    *result = Z3;
     return r;
 }
 
@@ -1204,11 +1198,11 @@ Parament_ErrorCode run(Context<R>* h, const cplx<R>* carr_dev, double dt, unsign
     C* leaves = nullptr;
     C* spare = nullptr;   // a buffer free for the other half of the tree's ping-pong
     if (ps.deg) {
-        C* w[4];
-        for (int i = 0; i < 4; ++i) w[i] = reinterpret_cast<C*>(gen[1 + i]);
-        if (poly_batched<R>(sizeof(R) == 8 ? pa::GEMM_F64 : pa::GEMM_F32, ps, X, (int)d, N, true, w, nullptr, &leaves,
-                            st) != hipSuccess)
-            return PARAMENT_STATUS_CUBLAS_FAILED;
+        if constexpr (sizeof(R) == 8) {
+            C* w[4];
+            for (int i = 0; i < 4; ++i) w[i] = reinterpret_cast<C*>(gen[1 + i]);
+            if (poly_batched(ps, X, (int)d, N, w, &leaves, st) != hipSuccess) return PARAMENT_STATUS_CUBLAS_FAILED;
+        }
         spare = X;
     } else if (power) {
         double mr[pa::kMaxCheb], mi[pa::kMaxCheb];

@@ -87,12 +87,17 @@ hipError_t launch_cheb_fused(const ChebArgs<R>& a, hipStream_t st) {
         return hipErrorInvalidValue;
     const int grid = a.N;
     if (a.pdeg) {
-        if (a.pdeg != 8 && a.pdeg != 12) return hipErrorInvalidValue;
-#define PA_POLY(DD)                                                                                                     \
-    if (a.pdeg == 8) hipLaunchKernelGGL((poly_fused_kernel<R, DD, 8>), dim3(grid), dim3(64 * Shape<DD>::G), 0, st, a); \
-    else hipLaunchKernelGGL((poly_fused_kernel<R, DD, 12>), dim3(grid), dim3(64 * Shape<DD>::G), 0, st, a);
-        if (a.d <= 16) { PA_POLY(16) } else if (a.d <= 32) { PA_POLY(32) } else if (a.d <= 48) { PA_POLY(48) }
-        else { PA_POLY(64) }
+        // complex64: the gradient's slices at M = 7 (dims up to 32)
+        if (sizeof(R) == 4 ? a.pdeg != 8 || a.d > 32 : a.pdeg != 8 && a.pdeg != 12) return hipErrorInvalidValue;
+#define PA_POLY(DD, DEG) hipLaunchKernelGGL((poly_fused_kernel<R, DD, DEG>), dim3(grid), dim3(64 * Shape<DD>::G), 0, st, a);
+#define PA_POLY2(DD) if (a.pdeg == 8) { PA_POLY(DD, 8) } else { PA_POLY(DD, 12) }
+        if constexpr (sizeof(R) == 4) {
+            if (a.d <= 16) { PA_POLY(16, 8) } else { PA_POLY(32, 8) }
+        } else {
+            if (a.d <= 16) { PA_POLY2(16) } else if (a.d <= 32) { PA_POLY2(32) } else if (a.d <= 48) { PA_POLY2(48) }
+            else { PA_POLY2(64) }
+        }
+#undef PA_POLY2
 #undef PA_POLY
         return hipGetLastError();
     }
