@@ -320,3 +320,23 @@ def test_ensemble_values_beyond_fp16(x, m, kind, others):
                 assert rel_err(u, ref) < 1e-3, dims[i]
         else:
             assert rel_err(u, ref) < 2e-5 + 2.0 ** -23 * pts[i] * x, dims[i]
+
+
+@pytest.mark.parametrize("x, m", [(0.1, 5), (0.4, 7), (0.9, 9)])
+@pytest.mark.parametrize("pts", [[1, 9, 300, 64, 2, 1000], [4100, 700, 4097, 513, 66, 4101]])
+def test_ensemble_split_slices_rounding(x, m, pts):
+    """The fp16 split slice kernel of the classes 32, 48 and 64 at controls of modulus 1: its constants and first-order
+    terms are FP64, so what is left against the degree-M polynomial are roundings of products (2^-22, of nodes
+    up to 2 in norm), which add up as sqrt(n), and the table's truncation (0.05 eps a slice at M = 7, where
+    the kernel's polynomial is a higher one): no constant part that grows with n x."""
+    from parament_amd.ensemble import Ensemble
+    dims, amps = [17, 32, 33, 48, 49, 64], [1, 3, 4, 2, 5, 1]
+    hs, cs = make_ensemble(92, dims, amps, pts, None)
+    dt = [x / eo.hamiltonian_norm(h[0], h[1:]) for h in hs]
+    with Ensemble(dims, amps, pts, dt, "none") as e:
+        e.set_hamiltonians(hs)
+        us = e.equiprop(cs)
+    for i, (h, c) in enumerate(zip(hs, cs)):
+        h0, hk, c32 = as_c64_inputs(h[0], h[1:], c)
+        ref = eo.equiprop(h0, hk, c32, dt[i], cycles=m)
+        assert rel_err(us[i], ref) < 2.0 ** -21 * pts[i] ** 0.5 + (0.05 * 2.0 ** -23 * pts[i] if m == 7 else 0), (dims[i], pts[i])

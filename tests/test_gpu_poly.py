@@ -285,3 +285,48 @@ def test_host_arrays_of_changing_length(prec, d):
             p.equiprop_device(dt, carr.data_ptr(), n, 2, out.data_ptr())
             p.synchronize()
             assert np.array_equal(u, out.cpu().numpy()), n
+
+
+@pytest.mark.parametrize("d, amps, n", [(2, 1, 1), (4, 2, 257), (3, 3, 16385), (8, 2, 40000), (5, 5, 4097), (8, 4, 64)])
+@pytest.mark.parametrize("x", [0.1, 0.3, 0.9, 1.4])
+def test_small_dims_rounding_complex64(d, amps, n, x):
+    """complex64 at dims up to 8 against the recurrence with the kernel's own FP32 constants, evaluated in 64 bits:
+    what is left are the roundings of single operations, M + 2 of them a slice at 2^-24 of E = O(x), which
+    differ from slice to slice (random controls) and add up as sqrt(n), twice that allowed; and the tree's, below
+    2^-20 in all."""
+    import parament_amd as parament
+    from tests.helpers import as_c64_inputs
+    h0, hks, c, dt = problem(d, amps, n, x, False)
+    with parament.Parament("fp32") as p:
+        p.set_hamiltonian(h0, *hks)
+        u = p.equiprop(dt, *c)
+        m = p.iteration_cycles
+    h0, hks, c = as_c64_inputs(h0, hks, c)
+    hnorm = eo.hamiltonian_norm(h0, hks)
+    a = eo.bessel_coefficients(m, dt * hnorm)
+    a0 = complex(np.complex64(a[0] - 1)) + 1
+    a = np.concatenate([[a0], a[1:].astype(np.complex64).astype(complex)])
+    s = float(np.float32(2 / hnorm))
+    r = eo.clenshaw(eo.assemble(h0, hks, c), a, 2 / s)
+    ref = eo.pairwise_tree(r)
+    assert rel_err(u, ref) < 2 * (m + 2) * 2.0 ** -24 * x * n ** 0.5 + 2.0 ** -20
+
+
+@pytest.mark.parametrize("d, n", [(192, 116), (256, 66)])
+def test_complex128_tiles_gradient(d, n):
+    """The gradient's two-product launches on 64-wide FP64 tiles against fourth-order differences of the oracle's
+    fidelity along a random direction (truncation below 1e-12, 1e-14 / h = 1e-10 of rounding): 1e-8."""
+    import parament_amd as parament
+    h0, hks, c, dt = problem(d, 2, n, 0.1, False)
+    rng = np.random.default_rng(d)
+    with parament.Parament("fp64") as p:
+        p.set_hamiltonian(h0, *hks)
+        target = p.equiprop(dt, *(c + 0.5))
+        f, g = p.gate_fidelity_gradient(dt, *c, target=target)
+        m = p.iteration_cycles
+    v, h = rng.uniform(-1, 1, c.shape), 1e-4
+    fid = lambda x: abs(np.sum(target.conj() * eo.equiprop(h0, hks, x, dt, cycles=m))) ** 2 / d ** 2
+    assert abs(f - fid(c)) < 1e-12
+    ref = (8 * (fid(c + h * v) - fid(c - h * v)) - (fid(c + 2 * h * v) - fid(c - 2 * h * v))) / (12 * h)
+    assert abs(ref) > 1e-4   # a direction in which F changes
+    assert abs(np.sum(g * v) - ref) < 1e-8
