@@ -165,7 +165,8 @@ LIBSPEC Parament_ErrorCode Parament_setPrecisionMode_fp64(Parament_Context_f64 *
 LIBSPEC int Parament_getPrecisionMode(Parament_Context_f32 *handle);
 LIBSPEC int Parament_getPrecisionMode_fp64(Parament_Context_f64 *handle);
 
-/* Chebyshev order M used by the last successful equiprop (-1 before any). */
+/* Chebyshev order M used by the last successful equiprop (-1 before any): the table's choice or the caller's.
+ * Where the table chose it, the polynomial evaluated may be of a higher degree (see the precision modes). */
 LIBSPEC int Parament_getIterationCycles(Parament_Context_f32 *handle);
 LIBSPEC int Parament_getIterationCycles_fp64(Parament_Context_f64 *handle);
 
@@ -270,7 +271,13 @@ LIBSPEC size_t Parament_getGradientWorkspace_fp64(Parament_Context_f64 *handle);
  * mode (FP32 throughout, FP32 iteration-count table, the power form where that mode takes it,
  * same quadrature and product order), except that where tau Hnorm <= 1 and M >= 5 instances of dim
  * 17 to 64 run their slices and lowest tree levels, and larger ones the power form's products and
- * their product tree, on scaled fp16 two-way splits (FP32-accurate, as the default mode).  setExecution(0) (default) runs the whole ensemble as
+ * their product tree, on scaled fp16 two-way splits (operands of 22 bits, FP32 accumulation).  Up to
+ * dim 64 that is so where the class (17-32, 33-48, 49-64) has 4,096 such slices or more, or needs one
+ * slice kernel for all its instances; otherwise, and with setExecution(1), these dims run in FP32.  An
+ * instance's last bits thus depend on the other instances of its class.  Slices whose values leave
+ * fp16's range (controls well above 1 in modulus, non-unitary ones) are formed again in FP32 up to
+ * dim 64; above, entries of 4 and more overflow, as in the default mode of a complex64 context.
+ * setExecution(0) (default) runs the whole ensemble as
  * one captured HIP graph: the instances of dim <= 64 in multi-instance kernels per dim class
  * (16, 32, 48, 64), the larger ones on batched GEMMs, on concurrent branches (up to four for the
  * larger ones); the tree block size and grid of each class are tuned on first use (or by

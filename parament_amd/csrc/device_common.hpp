@@ -122,7 +122,9 @@ template <class R, int TM, int TN> struct CTile {
 
 // FP64 complex products on three real ones, Ar Br, Ai Bi and (Ar + Ai)(Br + Bi): the FP64 matrix cores bound
 // every kernel that calls this, and the two additions per operand pair run on the vector units beside
-// them.  Normwise as accurate as four products.  (8,192 dim-64 slices and their tree 1.78 -> 1.66 ms.)
+// them.  Normwise as accurate as four products, not element by element: the imaginary part is a difference of terms twice
+// its size.  Propagators and gradients came out no further from 64 bits than with four in the mean (0.95 to 1.02 times, over
+// dims 2-200, 1 to 1,000 steps, M = 5 to 11, schemes included).  (8,192 dim-64 slices and their tree 1.78 -> 1.66 ms.)
 template <class R, int TM, int TN> struct C3Tile {
     typename Mma<R>::acc x[TM][TN], y[TM][TN], s[TM][TN];
     __device__ __forceinline__ void zero() {

@@ -9,14 +9,16 @@
 // with S = 2^14, h0 = fp16(x S), h1 = fp16(x S - h0), 22 bits in all; the three products
 // h0 h0', h0 h1', h1 h0' accumulated in FP32 and the sum scaled by 2^-28; operand entries must
 // stay below 4 in modulus, which holds for the power form's operands and the tree's deviations
-// from identity).  The epilogue is evaluated in FP64 and rounded once to the output type,
-// so a Clenshaw step's a_k I is added exactly.  Used for the Chebyshev steps
+// from identity).  The epilogue is evaluated in FP64 (FP32 for the fp16 split) and rounded once to the output
+// type, so a Clenshaw step's a_k I is added exactly.  Used for the Chebyshev steps
 // (parament.cpp:569-652) and the product-tree levels (parament.cpp:657-718) at dims where a
 // slice does not fit on chip.
 //
 // Tiling: a work-group computes a 64x64 output tile with 4 waves of 32x32 (2x2 blocks of
-// 16x16), or a 32x32 tile with 4 waves of 16x16 (less padding for dims just above a multiple
-// of 64); K advances in chunks of 32 staged in LDS (zero-padded past d).  Work items (batch b,
+// 16x16; FP64: 8 waves of 32x16), or a 32x32 tile with 4 waves of 16x16 (narrow launches, and less padding for
+// dims just above a multiple of 64); K advances in chunks of 32 (FP64: 16) staged in LDS (zero-padded past d).  Two
+// kernels of their own: whole FP32 products at some dims (zgemm_row_kernel), 128x128 tiles on a persistent grid for
+// the fp16 split (zgemm_f16_kernel).  Work items (batch b,
 // tile t) are assigned so that every XCD receives a contiguous range of them: the tiles of one
 // slice then share that XCD's L2 for their A rows and B columns.
 #include "kernels.hpp"

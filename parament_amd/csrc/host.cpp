@@ -853,7 +853,7 @@ template <class R> int gen_buffers(Context<R>* h, Workspace& ws, size_t bytes, i
 }
 
 // Step-wise form (any dim): the Clenshaw GEMMs (or the power form's) batched over all slices on
-// complex64 data with the products of the context's mode, every GEMM epilogue in FP64.  In the
+// complex64 data with the products of the context's mode, GEMM epilogues in FP64 (the fp16 split's in FP32).  In the
 // default mode the power form runs on scaled fp16 two-way split products (its operands Y = tau X,
 // S = Y^2, the Horner brackets and the tree's deviations stay below 4 in modulus while
 // ||tau X_j||_2 <= 1, as in the fused kernel), the recurrence on bf16 three-way splits.
@@ -1309,8 +1309,8 @@ template <class R> Parament_ErrorCode ensure_common(Context<R>* h, unsigned amps
 // Host-array calls stage controls of up to kPinIn bytes and results of up to kPinOut in pinned memory, which the
 // kernels read and write across the bus: a copy of either to or from the caller's pageable array takes 8 to 12 us,
 // more than a small problem's launches.  It is allocated as large as the arrays need (grow-only): 4 KB take 26 us, all of
-// it 42, in a context's first call.  Controls up to kPinDirect are read where they are by a one-launch
-// problem (each sample once); larger ones go to the device by a kernel.  Larger arrays take copies, whose
+// it 42, in a context's first call.  Controls up to kPinDirect are read where they are by the kernel of
+// dims up to 8 (each sample one to three times, by the quadrature); others go to the device by a kernel.  Larger arrays take copies, whose
 // rate is then what counts.
 constexpr size_t kPinIn = 512 << 10, kPinOut = 64 << 10, kPinDirect = 4 << 10;
 
@@ -2463,7 +2463,7 @@ hipError_t ens_enqueue(Ensemble* e) {
 }
 
 // Per-instance loop (the baseline the ensemble replaces): one problem after the other on one
-// stream with the single-problem kernels.
+// stream with the single-problem kernels, in FP32 up to dim 64 (also where the classes take the fp16 split).
 hipError_t ens_enqueue_loop(Ensemble* e) {
     hipError_t r = hipSuccess;
     for (size_t i = 0; r == hipSuccess && i < e->in.size(); ++i) {
@@ -2477,7 +2477,7 @@ hipError_t ens_enqueue_loop(Ensemble* e) {
         ca.ctl.mode = e->quad; ca.ctl.magnus = 0; ca.ctl.tau = (float)x.tau;
         for (int k = 0; k <= x.M; ++k) { ca.are[k] = (float)x.are[k]; ca.aim[k] = (float)x.aim[k]; }
         ca.are[0] = (float)(x.are[0] - 1.0);
-        if (stepwise_power(x.M, x.tau * x.hnorm)) {   // as the class kernels
+        if (stepwise_power(x.M, x.tau * x.hnorm)) {   // FP32 products, as the classes' FP32 kernels
             double mr[pa::kMaxCheb], mi[pa::kMaxCheb];
             power_coefficients(x.M, x.tau * x.hnorm, x.are, x.aim, mr, mi);
             ca.ps = 1;

@@ -120,8 +120,7 @@ template hipError_t launch_cheb_fused<float>(const ChebArgs<float>&, hipStream_t
 template hipError_t launch_cheb_fused<double>(const ChebArgs<double>&, hipStream_t);
 
 // ---------------------------------------------------------------------------------------
-// Dims 9-16 (and up to 8 with more coefficients than small.hip takes): one wave per work-group on a
-// persistent grid.  The operators are the
+// Dims 9-16 (smaller ones: small.hip): one wave per work-group on a persistent grid.  The operators are the
 // same for every slice, so they stay in LDS for the whole launch; each lane t < ncoef loads the
 // next slice's coefficient t while the current slice runs; and the F lowest tree levels are
 // folded on chip in the reference's pairing (binary counter, later node on the left, on

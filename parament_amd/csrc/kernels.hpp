@@ -98,15 +98,16 @@ template <class R> hipError_t launch_fill(const cplx<R>* X, cplx<R> alpha, cplx<
 hipError_t launch_assemble_c64(const ChebArgs<double>& a, float2* X, hipStream_t st);
 // n d x d complex64 matrices -> complex128.
 hipError_t launch_widen(const float2* in, int d, int n, double2* out, hipStream_t st);
-// n complex128 values -> complex64 (rounded to nearest).
+// bytes (a multiple of 8) from pinned host memory to the device, by a kernel.
 hipError_t launch_stage(const void* in, size_t bytes, void* out, hipStream_t st);
+// n complex128 values -> complex64 (rounded to nearest).
 hipError_t launch_narrow(const double2* in, long n, float2* out, hipStream_t st);
 // E_j = (a_0 - 1) I + a_1 s X_j + R_j in FP64 (are[0] = a_0 - 1), stored as complex64.
 hipError_t launch_first_order(const ChebArgs<double>& a, const float2* R, float2* E, hipStream_t st);
 
 // Batched complex GEMM on the matrix cores (gemm.hip), any dim:
 //     C_b = alpha A_b B_b + beta Cin_b + beta2 Cin2_b + diag I + ca A_b + cb B_b,
-// and, given D, a second output of the same product
+// and, given D, a second output of the same product (D, and ca, cb other than both 0 or both 1: complex128 only)
 //     D_b = d_ab A_b B_b + d_a A_b + d_b B_b + d_c Cin_b + d_c2 Cin2_b,
 // strides in matrices of d x d (0 broadcasts one matrix).  Element types: complex128 where the
 // flag is set, complex64 otherwise (Cin and Cin2 have C's type; C may be Cin or Cin2 itself).  GEMM_F64 needs a complex128 output and

@@ -514,8 +514,8 @@ __global__ __launch_bounds__(64 * HShape<D>::G, 2) void cheb_h2_kernel(MixedArgs
 
 // Nodes of many problems (an ensemble's dim class): task (i, w) is node w of inst[i], whose arguments stay
 // in memory and are read as scalars.  A node whose values leave fp16's range is formed again in FP32 products; those on
-// leading parts only, which rest on controls of modulus 1, are not used.  16 systems of dims 33-64 with 1,000-4,000 slices take 1.38 ms with it
-// against 2.42 ms on the FP32 slice kernel and its two lowest tree levels.
+// leading parts only, which rest on controls of modulus 1, are not used.  16 systems of dims 33-64 with
+// 1,000-4,000 slices take 1.41 ms with it against 2.42 ms on the FP32 slice kernel and its two lowest tree levels.
 template <int D, int F, int FULL, int SCHEME>
 __global__ __launch_bounds__(64 * HShape<D>::G, 2) void ens_h2_kernel(const MixedArgs* __restrict__ inst,
                                                                      const int2* __restrict__ tasks, int ntasks) {

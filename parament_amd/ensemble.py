@@ -2,8 +2,9 @@
 
 No counterpart in the reference package: many systems of different dimension, control count
 and length solved together.  Each instance gets what ``Parament('fp32').equiprop`` would return
-for it (same iteration-count table, quadrature and product order; FP32 products up to dim 64,
-FP32-accurate fp16 split products above, as the default mode's step-wise path); the ensemble
+for it (same iteration-count table, quadrature and product order; FP32 products up to dim 16, and where
+tau Hnorm > 1 or the order is below 5; fp16 two-way split products, 22 bits, at other dims, up to dim 64 for classes
+that are long enough or of one form, as ``parament.h`` states it); the ensemble
 runs as one captured HIP graph with multi-instance kernels for the small dims, batched GEMMs for
 dims above 64, concurrent branches and tuned tree block sizes and grids.
 """
@@ -122,7 +123,7 @@ class Ensemble:
 
     def set_execution(self, mode):
         """'graph' (default: multi-instance kernels in one captured graph) or 'loop' (one
-        instance after the other)."""
+        instance after the other, in FP32 up to dim 64)."""
         self._check(self._lib.Parament_ensembleSetExecution(self._handle, {"graph": 0, "loop": 1}[mode]))
 
     def tune(self):

@@ -243,7 +243,7 @@ class Parament:
 
     @property
     def iteration_cycles(self):
-        """Chebyshev order M used by the last successful :meth:`equiprop` (-1 before any)."""
+        """Chebyshev order M, chosen or set, of the last successful :meth:`equiprop` (-1 before any)."""
         if self._handle is None:
             return -1
         return self._call('Parament_getIterationCycles', self._handle)
